@@ -100,9 +100,11 @@ struct Reduced {
 // reduce_colors (icbc.h:1638-1683): texels of positive weight merge, in
 // texel order, into the first earlier cluster within 1/256 in every channel
 // (weighted running mean), or open a new one.  Leaves clusters 0..n-1 as
-// (r, g, b, weight) in rows[0..n-1].  Tame texels keep every product and sum
-// of the fits finite and normal (or an exact zero).  k: the block's known
-// cluster count (every texel of 16 clusters opens one).
+// (r, g, b, weight) in rows[0..n-1].  Tame texels, with weights of at most 1,
+// keep every sum and error of the searches finite, and those of unit weights
+// normal (or an exact zero) too; the principal axis, which squares its
+// covariances, they do not (lane_sat).  k: the block's known cluster count
+// (every texel of 16 clusters opens one).
 __device__ __forceinline__ Reduced lane_reduce(LaneRows rows, int lane, const BlockTexels &texels, int k)
 {
     const float thr = 1.0f / 256;
@@ -289,9 +291,12 @@ __device__ __forceinline__ float4 lane_sat(LaneRows rows, int lane, int n, bool 
         }
     }
     // The stable order by projection: ord[r], the cluster at rank r, in four
-    // bits each.
+    // bits each.  The keys below order numbers only, and tame texels have none
+    // where the axis squares covariances beyond the range of floats:
+    // components that lie 4e9 apart or more, weights of 1e-17 or less.
+    const bool axis = fabsf(vx) <= 1e18f && fabsf(vy) <= 1e18f && fabsf(vz) <= 1e18f;
     uint64_t ord = 0;
-    if (tame) {
+    if (tame && __builtin_amdgcn_ballot_w64(!axis) == 0) {
         // (projection, cluster) as doubles (TameBest; + 0 makes a -0 the 0
         // that the comparisons take it for), through an odd-even merge sort:
         // two instructions a comparator.  Ranks past n sort last.

@@ -217,6 +217,29 @@ def test_search_forms_match_one_pass(lanes, side, kind):
     assert _both_encoders(lanes, np.ascontiguousarray(img[:, :h]), w, h, **kw) == 0
 
 
+@pytest.mark.parametrize("side", [60, 1024])
+@pytest.mark.parametrize("scale, alpha", [(s, 1.0) for s in (1e8, 3e9, 1e10, 1e14, 9e17)] +
+                         [(1.0, a) for a in (1e-12, 1e-16, 1e-20, 1e-30)] + [(1e10, 1e-20)])
+def test_search_where_the_axis_overflows(lanes, oracle, side, scale, alpha):
+    """Components and weights whose sums and errors are finite, but whose
+    covariances have no finite squares, so that the projections that the
+    clusters are sorted by are NaN: blocks of 2 to 16 colours, the reference's
+    order (a NaN moves nothing) in both encoders."""
+    rng = np.random.default_rng(int(np.log10(scale)) * 7 + side)
+    nb = side // 4
+    pal = rng.random((nb, nb, 16, 3), dtype=np.float32) * np.float32(scale)
+    count = rng.integers(2, 17, (nb, nb, 1))
+    pick = np.where(rng.random((nb, nb, 1)) < 0.3, np.arange(16), rng.integers(0, 16, (nb, nb, 16))) % count
+    texels = np.take_along_axis(pal, pick[..., None], axis=2).reshape(nb, nb, 4, 4, 3)
+    img = np.empty((4, side, side), np.float32)
+    img[:3] = texels.transpose(4, 0, 2, 1, 3).reshape(3, side, side)
+    img[3] = np.float32(alpha)
+    kw = dict(alpha_mode=N.ALPHA_TRANSPARENCY)
+    assert _both_encoders(lanes, img, side, side, **kw) == 0
+    assert _diff(lanes.compress(N.FORMAT_BC1, img, side, side, **kw),
+                 oracle.compress(N.FORMAT_BC1, img.reshape(-1), side, side, **kw)) == 0
+
+
 def test_default_route_by_size_and_scratch():
     """A context as it is made: images and sets above the sizes where the
     two-pass encoder is optional, with and without a scratch limit (which
