@@ -193,7 +193,10 @@ NTX_API ntx_status ntx_hip_compress_device_noalloc(ntx_hip_context *ctx, int for
  * partials); a call that would exceed it allocates nothing and returns
  * NTX_ERR_OUT_OF_MEMORY (Error_CudaError in the nvtt front end, which then
  * goes on with the next image, as CudaCompressorDXT.cpp:183-189 does).
- * 0 = no cap (the default).  No counterpart in the reference. */
+ * Scratch that a call can do without (see ntx_hip_set_bc1_lanes_min) is given
+ * back when a cap is set, after the work on the context's stream, and not
+ * taken under one.  0 = no cap (the default).  No counterpart in the
+ * reference. */
 NTX_API ntx_status ntx_hip_set_scratch_limit(ntx_hip_context *ctx, size_t bytes);
 
 /* BC1 at icbc Level8 (Normal / Highest) has two encoders with identical

@@ -303,7 +303,7 @@ NTX_API ntx_status ntx_hip_destroy(ntx_hip_context *ctx)
     for (auto &kv : ctx->tail_taps) (void)hipFree(kv.second.packed);
     for (hipStream_t st : ctx->side)
         if (st) (void)hipStreamSynchronize(st);
-    for (DevBuf *b : { &ctx->in, &ctx->out, &ctx->tmp, &ctx->dst, &ctx->bucket, &ctx->metric, &ctx->chain })
+    for (DevBuf *b : { &ctx->in, &ctx->out, &ctx->tmp, &ctx->dst, &ctx->bucket, &ctx->metric, &ctx->chain, &ctx->optional })
         if (b->ptr) (void)hipFree(b->ptr);
     for (hipEvent_t e : ctx->sync_events) (void)hipEventDestroy(e);
     for (hipStream_t st : ctx->side)
@@ -760,10 +760,21 @@ static ntx_status single_bucket(ntx_hip_context *ctx, int format, int quality, i
     return NTX_OK;
 }
 
+// Gives the optional encoder's scratch back.  The searches that use it are on
+// the context's stream, and no graph holds it (optional_bc1_bucket).
+static hipError_t release_optional(ntx_hip_context *ctx)
+{
+    if (!ctx->optional.ptr) return hipSuccess;
+    hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = hipFree(ctx->optional.ptr);
+    if (e == hipSuccess) ctx->optional = {};
+    return e;
+}
+
 // Scratch for the two-pass BC1 encoder over `blocks` blocks that do not
-// require it, or null: none under a scratch limit, which other calls may
-// need, and none while the stream records a graph, which neither may allocate
-// nor keep this memory (a later call may move it).
+// require it (ctx->optional), or null: none under a scratch limit, which other
+// calls may need, and none while the stream records a graph, which neither may
+// allocate nor keep this memory (a later call may move it).
 static int *optional_bc1_bucket(ntx_hip_context *ctx, int quality, size_t blocks)
 {
     if (ctx->bc1_lanes_min != ntx_hip_context::kBc1LanesMinDefault || ctx->scratch_limit || bc1_level(quality) != 8 ||
@@ -771,16 +782,19 @@ static int *optional_bc1_bucket(ntx_hip_context *ctx, int quality, size_t blocks
         return nullptr;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
-    const size_t cap_before = ctx->bucket.cap;
-    const std::string err = ctx->err;
-    if (ensure(ctx, ctx->bucket, sizeof(int) * size_t(bc1_scratch_ints(int(blocks)))) != NTX_OK) {
-        // The device is full: the one-pass encoder does.
-        (void)hipGetLastError();
-        ctx->err = err;
-        return nullptr;
+    const size_t bytes = sizeof(int) * size_t(bc1_scratch_ints(int(blocks)));
+    if (ctx->optional.cap < bytes) {
+        void *p = nullptr;
+        if (release_optional(ctx) != hipSuccess || hipMalloc(&p, bytes) != hipSuccess) {
+            // The device is full: the one-pass encoder does.
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        ctx->optional.ptr = p;
+        ctx->optional.cap = bytes;
+        ctx->optional_counts_zero = false;  // fresh memory
     }
-    if (ctx->bucket.cap != cap_before) ctx->bc3_counts_zero = false;  // fresh memory
-    return static_cast<int *>(ctx->bucket.ptr);
+    return static_cast<int *>(ctx->optional.ptr);
 }
 
 // BC1 images at Level8 in one pair of launches (launch_bc1_set) on the
@@ -804,13 +818,13 @@ static hipError_t bc1_set_on(ntx_hip_context *ctx, int quality, int alpha_mode, 
     if (!bucket) return hipSuccess;
     *done = true;
     hipError_t e = hipSuccess;
-    if (!ctx->bc3_counts_zero) e = launch_bc3_clear_counts(bucket, ctx->stream);
-    ctx->bc3_counts_zero = false;
+    if (!ctx->optional_counts_zero) e = launch_bc3_clear_counts(bucket, ctx->stream);
+    ctx->optional_counts_zero = false;
     if (e == hipSuccess)
         e = timed_on(ctx, ctx->stream, NTX_KERNEL_BC1_SEARCH, [&] {
             return launch_bc1_set(t, n, alpha_mode, cw, ctx->d_tab, bucket, int(blocks), ctx->cus, ctx->stream);
         });
-    if (e == hipSuccess) ctx->bc3_counts_zero = true;
+    if (e == hipSuccess) ctx->optional_counts_zero = true;
     return e;
 }
 
@@ -830,11 +844,14 @@ NTX_API ntx_status ntx_hip_compress_device(ntx_hip_context *ctx, int format, int
     if (!cw) cw = ones;
     int *bucket = nullptr;
     if ((s = ntx::single_bucket(ctx, format, quality, w, h, &bucket))) return s;
+    bool *counts_zero = &ctx->bc3_counts_zero;
     const size_t blocks = size_t((w + 3) / 4) * size_t((h + 3) / 4);
-    if (!bucket && format == NTX_FORMAT_BC1 && blocks >= size_t(ntx_hip_context::kBc1LanesOptional))
+    if (!bucket && format == NTX_FORMAT_BC1 && blocks >= size_t(ntx_hip_context::kBc1LanesOptional)) {
         bucket = ntx::optional_bc1_bucket(ctx, quality, blocks);
+        counts_zero = &ctx->optional_counts_zero;
+    }
     hipError_t e = ntx::compress_on(ctx, ctx->stream, format, quality, alpha_mode, cw, d_rgba, w, h, d_out, bucket,
-                                    &ctx->bc3_counts_zero);
+                                    counts_zero);
     if (e != hipSuccess) return fail(ctx, e, "compress launch");
     return NTX_OK;
 }
@@ -843,6 +860,10 @@ NTX_API ntx_status ntx_hip_set_scratch_limit(ntx_hip_context *ctx, size_t bytes)
 {
     if (!ctx) return NTX_ERR_INVALID_ARGUMENT;
     ctx->scratch_limit = bytes;
+    if (bytes && ctx->optional.ptr) {
+        if (ntx_status s = bind(ctx)) return s;
+        NTX_HIP(ctx, ntx::release_optional(ctx));
+    }
     return NTX_OK;
 }
 

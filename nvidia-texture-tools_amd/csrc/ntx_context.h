@@ -173,6 +173,12 @@ struct ntx_hip_context {
     // The BC3 tallies at the start of `bucket` are zero: set after a complete
     // front + search sequence (the search clears them), cleared before one.
     bool bc3_counts_zero = false;
+    // The optional two-pass encoder's scratch and whether its tallies are
+    // zero.  Apart from the buffers above, so that a call that does without it
+    // neither moves memory that a recorded graph holds nor counts towards a
+    // scratch limit set later, which also gives it back.
+    ntx::DevBuf optional;
+    bool optional_counts_zero = false;
     // Concurrent compression of several images (mip chains, image sets):
     // the side streams, fork/join events, and per-image BC3 scratch (every
     // region's tallies zero when chain_counts_zero).

@@ -6,6 +6,7 @@ checks are the same as for the one-pass encoder: the reference icbc's golden
 blocks, the oracle on adversarial blocks and seeded images (byte for byte),
 the per-block colour counts (n, m) against the oracle's, and the two
 encoders against each other on larger images."""
+import ctypes
 import os
 
 import numpy as np
@@ -268,3 +269,83 @@ def test_default_route_by_size_and_scratch():
     finally:
         for ctx in (free, capped, one):
             ctx.close()
+
+
+class _Capture:
+    """HIP stream capture through the library's own runtime: mode 0 global, 2 relaxed."""
+
+    def __init__(self, ctx, stream, mode):
+        self.lib, self.stream, self.graph, self.exec = ctx.lib, ctypes.c_void_p(stream), ctypes.c_void_p(), ctypes.c_void_p()
+        self.mode = mode
+
+    def __enter__(self):
+        assert self.lib.hipStreamBeginCapture(self.stream, self.mode) == 0
+        return self
+
+    def __exit__(self, *exc):
+        assert self.lib.hipStreamEndCapture(self.stream, ctypes.byref(self.graph)) == 0
+        if exc[0] is None and self.graph:
+            assert self.lib.hipGraphInstantiate(ctypes.byref(self.exec), self.graph, None, None, ctypes.c_size_t(0)) == 0
+
+    def launch(self):
+        assert self.lib.hipGraphLaunch(self.exec, self.stream) == 0
+
+    def close(self):
+        for f, h in ((self.lib.hipGraphExecDestroy, self.exec), (self.lib.hipGraphDestroy, self.graph)):
+            if h:
+                assert f(h) == 0
+
+
+def _input(ctx, w, h, seed):
+    p = synth.to_planar(synth.noise_rect_rgba(w, h, seed=seed)).reshape(-1)
+    return p, ctx.alloc(p.nbytes).upload(p)
+
+
+def test_optional_scratch_is_off_a_later_limit():
+    """Calls that took the two-pass encoder's optional scratch leave a limit
+    that is set afterwards to the calls that need theirs."""
+    with N.Context(0) as ctx:
+        w, h = 1000, 917
+        _, d = _input(ctx, w, h, 81)
+        _, d2 = _input(ctx, 640, 480, 82)
+        out = [ctx.alloc(N.compressed_size(N.FORMAT_BC1, a, b)) for a, b in ((w, h), (640, 480))]
+        ctx.compress_images_device(N.FORMAT_BC1, [d, d2], [(w, h), (640, 480)], out)
+        ctx.compress_device(N.FORMAT_BC1, d, w, h, out[0])
+        first = out[0].download(np.uint8)
+        small = synth.to_planar(synth.noise_rect_rgba(64, 64, seed=83)).reshape(-1)
+        ctx.lib.ntx_hip_set_scratch_limit(ctx.handle, small.nbytes + N.compressed_size(N.FORMAT_BC4, 64, 64))
+        ctx.compress(N.FORMAT_BC4, small, 64, 64)
+        for limit in (1, 0, 1 << 30, 0):  # without it, with it, and back
+            ctx.lib.ntx_hip_set_scratch_limit(ctx.handle, limit)
+            out[0].upload(np.zeros_like(first))
+            ctx.compress_device(N.FORMAT_BC1, d, w, h, out[0])
+            assert np.array_equal(out[0].download(np.uint8), first), limit
+
+
+def test_optional_scratch_and_recorded_graphs():
+    """A graph recorded over a call that needs the context's scratch, replayed
+    after calls that took the optional one and between others."""
+    with N.Context(0) as ctx:
+        w, h = 128, 96
+        _, d = _input(ctx, w, h, 91)
+        _, big = _input(ctx, 1000, 917, 92)
+        out = ctx.alloc(N.compressed_size(N.FORMAT_BC3, w, h))
+        out_big = ctx.alloc(N.compressed_size(N.FORMAT_BC1, 1000, 917))
+        ctx.compress_device(N.FORMAT_BC3, d, w, h, out)  # its scratch is there before the recording
+        want = out.download(np.uint8)
+        with _Capture(ctx, ctx.lib.ntx_hip_stream(ctx.handle), 2) as g:
+            ctx.compress_device(N.FORMAT_BC3, d, w, h, out)
+        results = []
+        for k in range(4):
+            if k:
+                ctx.compress_device(N.FORMAT_BC1, big, 1000, 917, out_big)
+                results.append(out_big.download(np.uint8))
+            out.upload(np.zeros_like(want))
+            g.launch()
+            ctx.synchronize()
+            assert np.array_equal(out.download(np.uint8), want), k
+        ctx.set_bc1_lanes_min(1 << 30)
+        ctx.compress_device(N.FORMAT_BC1, big, 1000, 917, out_big)
+        for r in results:
+            assert np.array_equal(r, out_big.download(np.uint8))
+        g.close()
