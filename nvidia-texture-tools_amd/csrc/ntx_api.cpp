@@ -68,9 +68,26 @@ hipEvent_t take_event(ntx_hip_context *ctx)
 }
 
 
+// While one of these lives, this thread may allocate although some other
+// stream of the process records a graph, for the sake of calls that have
+// nothing else to do with such a recording.
+class AnyCapture {
+public:
+    AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    ~AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    AnyCapture(const AnyCapture &) = delete;
+    AnyCapture &operator=(const AnyCapture &) = delete;
+
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 ntx_status host_result(ntx_hip_context *ctx, void **p)
 {
-    if (!ctx->host_result) NTX_HIP(ctx, hipHostMalloc(&ctx->host_result, kHostResultBytes, hipHostMallocDefault));
+    if (!ctx->host_result) {
+        const AnyCapture allow;
+        NTX_HIP(ctx, hipHostMalloc(&ctx->host_result, kHostResultBytes, hipHostMallocDefault));
+    }
     *p = ctx->host_result;
     return NTX_OK;
 }
@@ -765,6 +782,7 @@ static ntx_status single_bucket(ntx_hip_context *ctx, int format, int quality, i
 static hipError_t release_optional(ntx_hip_context *ctx)
 {
     if (!ctx->optional.ptr) return hipSuccess;
+    const AnyCapture allow;
     hipError_t e = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) e = hipFree(ctx->optional.ptr);
     if (e == hipSuccess) ctx->optional = {};
@@ -784,6 +802,7 @@ static int *optional_bc1_bucket(ntx_hip_context *ctx, int quality, size_t blocks
     if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
     const size_t bytes = sizeof(int) * size_t(bc1_scratch_ints(int(blocks)));
     if (ctx->optional.cap < bytes) {
+        const AnyCapture allow;
         void *p = nullptr;
         if (release_optional(ctx) != hipSuccess || hipMalloc(&p, bytes) != hipSuccess) {
             // The device is full: the one-pass encoder does.

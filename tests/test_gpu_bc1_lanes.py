@@ -324,7 +324,9 @@ def test_optional_scratch_is_off_a_later_limit():
 
 def test_optional_scratch_and_recorded_graphs():
     """A graph recorded over a call that needs the context's scratch, replayed
-    after calls that took the optional one and between others."""
+    after calls that took the optional one and between others; and a call with
+    the optional scratch while another stream records, which the recording
+    survives."""
     with N.Context(0) as ctx:
         w, h = 128, 96
         _, d = _input(ctx, w, h, 91)
@@ -335,10 +337,17 @@ def test_optional_scratch_and_recorded_graphs():
         want = out.download(np.uint8)
         with _Capture(ctx, ctx.lib.ntx_hip_stream(ctx.handle), 2) as g:
             ctx.compress_device(N.FORMAT_BC3, d, w, h, out)
+        other = ctypes.c_void_p()
+        assert ctx.lib.hipStreamCreateWithFlags(ctypes.byref(other), 1) == 0
+        recording = _Capture(ctx, other.value, 0)
         results = []
         for k in range(4):
-            if k:
+            if k == 1:
+                with recording:
+                    ctx.compress_device(N.FORMAT_BC1, big, 1000, 917, out_big)
+            elif k > 1:
                 ctx.compress_device(N.FORMAT_BC1, big, 1000, 917, out_big)
+            if k:
                 results.append(out_big.download(np.uint8))
             out.upload(np.zeros_like(want))
             g.launch()
@@ -349,3 +358,5 @@ def test_optional_scratch_and_recorded_graphs():
         for r in results:
             assert np.array_equal(r, out_big.download(np.uint8))
         g.close()
+        recording.close()
+        assert ctx.lib.hipStreamDestroy(other) == 0
