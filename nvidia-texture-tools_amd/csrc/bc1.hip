@@ -32,25 +32,39 @@ struct Bc1Jobs {
     int n;
     Bc1Job job[ntx::kBc1MaxImages];
 };
+// The image of a workgroup.
+__device__ __forceinline__ const Bc1Job &job_of(const Bc1Job &job, int) { return job; }
+__device__ __forceinline__ const Bc1Job &job_of(const Bc1Jobs &jobs, int group)
+{
+    int j = 0;
+    while (j + 1 < jobs.n && group >= jobs.job[j + 1].first) j++;
+    return jobs.job[j];
+}
 
-template <int LEVEL>
-__global__ __launch_bounds__(256) void bc1_kernel(Bc1Jobs jobs, int alpha_mode, float cwx, float cwy, float cwz,
+// Jobs: Bc1Job, one image, whose fields are loaded together at the start, or
+// Bc1Jobs.
+//
+// Level 9 is held to eight wavefronts a SIMD (64 registers, without spills);
+// left to itself the compiler takes 84 for one image and 64 to 66 for several,
+// with every size slower: Production of 700 x 300, 2048^2 and 4096^2 136,
+// 1,242 and 4,120 us with 84 of them, 128, 1,178 and 3,775 us so.  Level 8 has
+// the LDS of its term tables for four; Level 1 is left alone (held to eight
+// 8192^2 takes 1,645 us, not 1,600).
+template <int LEVEL, class Jobs>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LEVEL == 9 ? 8 : LEVEL == 8 ? 4 : 1)))
+void bc1_kernel(Jobs jobs, int alpha_mode, float cwx, float cwy, float cwz,
                                                   const ntx::Tables *__restrict__ tab, int urgent)
 {
     if (urgent) __builtin_amdgcn_s_setprio(3);
     __shared__ Bc1Shared sh;
     __shared__ TermTables s_terms;
-    int j = 0;
-    while (j + 1 < jobs.n && int(blockIdx.x) >= jobs.job[j + 1].first) j++;
-    const Bc1Job &im = jobs.job[j];
+    const Bc1Job &im = job_of(jobs, int(blockIdx.x));
     const int g = threadIdx.x >> 4;
     const int lane = threadIdx.x & 15;
-    const int parts = im.parts;
+    const int parts = LEVEL == 8 ? im.parts : 1;
     // A block on a whole workgroup searches in five trips: fewer than the
-    // term tables' 18 KB are worth.  Level 9 spends its time in the refinement,
-    // which the tables' LDS and registers leave four wavefronts a SIMD where
-    // it has seven without them (2048^2: 1,277 us with them, 1,200 without;
-    // held to eight it is 5 us less there, but 700 x 300 takes 132 us, not 127).
+    // term tables' 18 KB are worth.  Level 9 spends its time in the refinement
+    // and wants the wavefronts that the tables would cost it.
     const bool use_terms = LEVEL == 8 && parts < kBlocksPerWG;
     load_shared_tables(sh, tab, threadIdx.x, blockDim.x);
     if (use_terms) load_term_tables(s_terms, tab, threadIdx.x, blockDim.x);
@@ -520,9 +534,14 @@ hipError_t launch_bc1(const Bc1Target *images, int n, int alpha_mode, const floa
         jobs.n++;
     }
     if (jobs.n == 0) return hipSuccess;
-    auto kernel = level == 1 ? bc1_kernel<1> : level == 9 ? bc1_kernel<9> : bc1_kernel<8>;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlocksPerWG * kGroup), 0, stream, jobs, alpha_mode, cw[0], cw[1], cw[2],
-                       d_tab, urgent ? 1 : 0);
+    auto launch = [&](auto kernel, const auto &args) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlocksPerWG * kGroup), 0, stream, args, alpha_mode, cw[0], cw[1],
+                           cw[2], d_tab, urgent ? 1 : 0);
+    };
+    if (jobs.n == 1)
+        launch(level == 1 ? bc1_kernel<1, Bc1Job> : level == 9 ? bc1_kernel<9, Bc1Job> : bc1_kernel<8, Bc1Job>, jobs.job[0]);
+    else
+        launch(level == 1 ? bc1_kernel<1, Bc1Jobs> : level == 9 ? bc1_kernel<9, Bc1Jobs> : bc1_kernel<8, Bc1Jobs>, jobs);
     return hipGetLastError();
 }
 
