@@ -913,6 +913,8 @@ static hipError_t bc1_images_on(ntx_hip_context *ctx, hipStream_t stream, int qu
     return e;
 }
 
+constexpr size_t kBc1ApartLevel9 = 3 << 16;  // see compress_many
+
 // n independent images compressed concurrently, in the caller's order (the
 // largest first).  BC1 images at Level8 share the two-pass encoder's launches
 // where bc1_set_on applies.  Where it does not, those of the one-pass encoder
@@ -943,6 +945,17 @@ static ntx_status compress_many(ntx_hip_context *ctx, int format, int quality, i
     int apart = n;
     if (format == NTX_FORMAT_BC1)
         while (apart > 0 && !bc1_two_pass(ctx, quality, w[apart - 1], h[apart - 1])) apart--;
+    // So have the three largest of a large set at Level9, whose blocks take 100
+    // us or so: in one launch the small images' are the last to start, a tail
+    // behind all others.  In a small set that tail is shorter than what the side
+    // streams' forks and joins add (chains, all in one launch and three apart:
+    // 1024^2, 87,400 blocks, 404 and 436 us; 1500^2, 187,500, 652 and 662;
+    // 2048^2, 349,500, 1,560 and 1,500; 4096^2 of sRGB texels made linear 5,000
+    // and 4,820).
+    size_t blocks = 0;
+    for (int k = 0; k < n; k++) blocks += size_t((w[k] + 3) / 4) * size_t((h[k] + 3) / 4);
+    if (format == NTX_FORMAT_BC1 && bc1_level(quality) == 9 && blocks >= kBc1ApartLevel9)
+        apart = std::max(apart, std::min(n, 3));
     if (apart == 0) {
         const hipError_t e = bc1_images_on(ctx, ctx->stream, quality, alpha_mode, cw, n, d_in, w, h, d_out, false);
         return e == hipSuccess ? NTX_OK : fail(ctx, e, "compress launch");

@@ -133,3 +133,25 @@ def test_batch_mixing_qualities(gpu, oracle):
                 assert np.array_equal(b.blocks(t, k), exp), (t, k)
     for d in bufs:
         d.free()
+
+
+@pytest.mark.parametrize("quality", [PROD, FAST])
+@pytest.mark.parametrize("sizes", [[(1024, 1024)] * 2, [(1792, 1760)], [(64, 36), (1792, 1760)], [(1, 1), (1792, 1756), (7, 9)],
+                                   [(300, 200), (1792, 1756), (256, 64), (4, 3)] + [(60, 20)] * 17],
+                         ids=["two_below", "one", "two", "three", "many"])
+def test_image_sets_as_single_images(gpu, quality, sizes):
+    """Sets around 196,608 blocks (131,072 in all; 197,120 and more), where
+    Production's three first images get launches of their own, in any order
+    of size, with more images than a launch takes: every image's bytes are
+    those of a call of its own."""
+    d = [gpu.alloc(16 * w * h).upload(synth.to_planar(synth.noise_rect_rgba(w, h, seed=200 + k)).reshape(-1))
+         for k, (w, h) in enumerate(sizes)]
+    out = [gpu.alloc(N.compressed_size(N.FORMAT_BC1, w, h)) for w, h in sizes]
+    gpu.compress_images_device(N.FORMAT_BC1, d, sizes, out, quality=quality)
+    got = [o.download(np.uint8) for o in out]
+    for k, (w, h) in enumerate(sizes):
+        out[k].upload(np.zeros_like(got[k]))
+        gpu.compress_device(N.FORMAT_BC1, d[k], w, h, out[k], quality=quality)
+        assert np.array_equal(out[k].download(np.uint8), got[k]), k
+    for b in d + out:
+        b.free()
