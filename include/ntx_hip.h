@@ -115,8 +115,8 @@ enum {
     NTX_KERNEL_BC3_SEARCH_SPLIT = 14, /* BC3 colour search of a small image: 2..64 lanes per block */
     NTX_KERNEL_GAMMA = 15,       /* gamma transforms of R, G, B (one launch per up to 16 levels) */
     NTX_KERNEL_NORMALS = 16,     /* normal-map renormalisation of a generated level */
-    NTX_KERNEL_BC1_CLASSIFY = 17, /* BC1 pass 1 (large images): colour counts, 0/1-colour blocks, bucketing */
-    NTX_KERNEL_BC1_SEARCH = 18,  /* BC1 pass 2: cluster fit, one block per lane, over the buckets */
+    NTX_KERNEL_BC1_CLASSIFY = 17, /* BC1 pass 1 (large images and sets): colour counts, 0/1-colour blocks, bucketing */
+    NTX_KERNEL_BC1_SEARCH = 18,  /* BC1 pass 2: cluster fit, 1 to 8 lanes per block, over the buckets */
     NTX_KERNEL_OPTIMAL_CHANNEL = 19, /* OptimalCompress::compressDXT5A, 16 lanes per channel block */
     NTX_KERNEL_OPTIMAL_GREEN = 20,   /* OptimalCompress::compressDXT1G (BC3n Highest colour), one wavefront per block */
     NTX_KERNEL_BC3_FAST = 21,        /* QuickCompress::compressDXT5 (BC3 / BC3n Fastest), one thread per block */

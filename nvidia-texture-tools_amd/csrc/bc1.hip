@@ -611,15 +611,10 @@ hipError_t launch_bc1_search_multi(const Bc1Image *d_imgs, int nimgs, const Tabl
     return launch_search(table, d_tab, nullptr, d_counts, d_lists, cap, cus, stream);
 }
 
-// Both passes over up to kBc1MaxImages images of at most
-// bc1_multi_max_blocks() blocks each, together `cap` blocks, in two launches;
-// d_counts: bucket scratch of bc1_scratch_ints(cap) ints with zero tallies,
-// which are zero again afterwards.
-hipError_t launch_bc1_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, const Tables *d_tab,
-                          int *d_counts, int cap, int cus, hipStream_t stream)
+static ImageSet image_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, int *chunks)
 {
     ImageSet set{};
-    int chunks = 0;
+    *chunks = 0;
     for (int k = 0; k < n && k < kBc1MaxImages; k++) {
         const Bc1Target &t = images[k];
         Bc1Image &im = set.imgs[k];
@@ -630,15 +625,35 @@ hipError_t launch_bc1_set(const Bc1Target *images, int n, int alpha_mode, const 
         im.alpha_mode = alpha_mode;
         im.rows16 = (reinterpret_cast<uintptr_t>(t.src) & 15) == 0 && (t.w & 3) == 0;
         for (int c = 0; c < 3; c++) im.cw[c] = cw[c];
-        set.first[k] = chunks;
-        chunks += (((t.w + 3) / 4) * ((t.h + 3) / 4) + 255) / 256;
+        set.first[k] = *chunks;
+        *chunks += (((t.w + 3) / 4) * ((t.h + 3) / 4) + 255) / 256;
         set.n = k + 1;
     }
+    return set;
+}
+
+// The two passes over up to kBc1MaxImages images of at most
+// bc1_multi_max_blocks() blocks each, together `cap` blocks, in a launch
+// each; d_counts: bucket scratch of bc1_scratch_ints(cap) ints with zero
+// tallies, which are zero again after the second.
+hipError_t launch_bc1_classify_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, const Tables *d_tab,
+                                   int *d_counts, int cap, hipStream_t stream)
+{
+    int chunks = 0;
+    const ImageSet set = image_set(images, n, alpha_mode, cw, &chunks);
     if (chunks == 0) return hipSuccess;
     int *d_lists = d_counts + ntx_bucket::kListsOffset;
     hipLaunchKernelGGL(bc1_classify_set_kernel, dim3(chunks), dim3(256), 0, stream, set, d_tab, d_counts, d_lists, cap);
-    const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? launch_search(set, d_tab, nullptr, d_counts, d_lists, cap, cus, stream) : e;
+    return hipGetLastError();
+}
+
+hipError_t launch_bc1_search_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, const Tables *d_tab,
+                                 int *d_counts, int cap, int cus, hipStream_t stream)
+{
+    int chunks = 0;
+    const ImageSet set = image_set(images, n, alpha_mode, cw, &chunks);
+    if (chunks == 0) return hipSuccess;
+    return launch_search(set, d_tab, nullptr, d_counts, d_counts + ntx_bucket::kListsOffset, cap, cus, stream);
 }
 
 // icbc Level8 of the *d_count blocks listed in d_list (at most cap, each

@@ -816,7 +816,7 @@ static int *optional_bc1_bucket(ntx_hip_context *ctx, int quality, size_t blocks
     return static_cast<int *>(ctx->optional.ptr);
 }
 
-// BC1 images at Level8 in one pair of launches (launch_bc1_set) on the
+// BC1 images at Level8 in one pair of launches (launch_bc1_classify_set) on the
 // context's stream, where that applies: few enough, none too large, together
 // enough blocks, and scratch to be had.  *done: they were enqueued.
 static hipError_t bc1_set_on(ntx_hip_context *ctx, int quality, int alpha_mode, const float *cw, int n,
@@ -840,8 +840,12 @@ static hipError_t bc1_set_on(ntx_hip_context *ctx, int quality, int alpha_mode, 
     if (!ctx->optional_counts_zero) e = launch_bc3_clear_counts(bucket, ctx->stream);
     ctx->optional_counts_zero = false;
     if (e == hipSuccess)
+        e = timed_on(ctx, ctx->stream, NTX_KERNEL_BC1_CLASSIFY, [&] {
+            return launch_bc1_classify_set(t, n, alpha_mode, cw, ctx->d_tab, bucket, int(blocks), ctx->stream);
+        });
+    if (e == hipSuccess)
         e = timed_on(ctx, ctx->stream, NTX_KERNEL_BC1_SEARCH, [&] {
-            return launch_bc1_set(t, n, alpha_mode, cw, ctx->d_tab, bucket, int(blocks), ctx->cus, ctx->stream);
+            return launch_bc1_search_set(t, n, alpha_mode, cw, ctx->d_tab, bucket, int(blocks), ctx->cus, ctx->stream);
         });
     if (e == hipSuccess) ctx->optional_counts_zero = true;
     return e;

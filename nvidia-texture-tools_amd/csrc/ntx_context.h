@@ -36,8 +36,10 @@ hipError_t launch_bc1_search_multi(const Bc1Image *d_imgs, int nimgs, const Tabl
 // searches: a grid-stride loop over the blocks.
 constexpr int kOptimalGroupsPerCU = 8;
 int bc1_scratch_ints(int nblocks);
-hipError_t launch_bc1_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, const Tables *d_tab,
-                          int *d_counts, int cap, int cus, hipStream_t stream);
+hipError_t launch_bc1_classify_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, const Tables *d_tab,
+                                   int *d_counts, int cap, hipStream_t stream);
+hipError_t launch_bc1_search_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, const Tables *d_tab,
+                                 int *d_counts, int cap, int cus, hipStream_t stream);
 hipError_t launch_channels(const float *d_src, int w, int h, int format, void *d_out, hipStream_t stream,
                            bool urgent = false);
 hipError_t launch_bc3_front(const float *d_src, int w, int h, const Tables *d_tab, void *d_out, int *d_counts,
