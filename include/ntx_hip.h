@@ -390,7 +390,8 @@ typedef struct {
     int channel_jobs_per_item; /* multiple of 256 (a BC5 block is two jobs) */
     int mip_tiles_per_item;
     int mip_tile_width;        /* 16, 32, 64, 128 or 256 outputs; tile height = 256 / width */
-    int kernel_variant;        /* 0: 4 waves/SIMD, 1: 5, 2: 6 (register budget of the kernel) */
+    int kernel_variant;        /* staged schedule: register budget for the compiler's choice (0), 5 (1) or 6 (2) waves/SIMD;
+                                  without effect in the one-launch schedule */
     int workgroups;            /* persistent workgroups, 0 = as many as are resident */
     int schedule;              /* 0: a launch per mip stage, then the persistent compression launch;
                                   1: mips and compression in one persistent launch */

@@ -269,13 +269,13 @@ __global__ __launch_bounds__(256) void batch_mip_kernel(BatchArgs a)
 // schedule, every level already complete.  kMips true: the one-launch
 // schedule, mip items included and dependencies waited for.
 // kWaves: waves per SIMD the register allocation is held to (0: the
-// compiler's choice); the autotuner picks among the instances.  The LDS of
-// the one-launch schedule admits four workgroups a compute unit, hence four
-// waves per SIMD, so its registers are held to those.  kTiers: the
+// compiler's choice); the autotuner picks among the staged schedule's
+// instances.  The LDS of the one-launch schedule admits four workgroups a
+// compute unit, hence four waves per SIMD.  kTiers: the
 // batch holds BC1 levels at icbc levels other than 8 (Fastest, Production),
 // whose code would otherwise cost every batch registers.
 template <int kWaves, bool kTiers, bool kMips>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMips ? 4 : kWaves > 0 ? kWaves : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves > 0 ? kWaves : 1)))
 void batch_kernel(BatchArgs a)
 {
     __shared__ ntx_bc1::Bc1Shared sh;
@@ -339,23 +339,18 @@ __global__ __launch_bounds__(256) void batch_reset_kernel(int *p, int n)
 
 namespace ntx {
 
-// variant 0-2: the tuned register budget (compiler's choice, 5 or 6 waves per
-// SIMD); tiers: the instance with the BC1 Fastest / Production paths; mips:
-// the one-launch schedule's instance.
+// variant 0-2: the staged schedule's register budget (compiler's choice, 5 or
+// 6 waves per SIMD); tiers: the instance with the BC1 Fastest / Production
+// paths; mips: the one-launch schedule, whose register budget is fixed.
 using BatchKernel = void (*)(BatchArgs);
-template <bool kMips>
-BatchKernel batch_kernel_sched(int variant, bool tiers)
-{
-    switch (variant) {
-    case 1: return tiers ? batch_kernel<5, true, kMips> : batch_kernel<5, false, kMips>;
-    case 2: return tiers ? batch_kernel<6, true, kMips> : batch_kernel<6, false, kMips>;
-    default: return tiers ? batch_kernel<0, true, kMips> : batch_kernel<0, false, kMips>;
-    }
-}
-
 BatchKernel batch_kernel_of(int variant, bool tiers, bool mips)
 {
-    return mips ? batch_kernel_sched<true>(variant, tiers) : batch_kernel_sched<false>(variant, tiers);
+    if (mips) return tiers ? batch_kernel<4, true, true> : batch_kernel<4, false, true>;
+    switch (variant) {
+    case 1: return tiers ? batch_kernel<5, true, false> : batch_kernel<5, false, false>;
+    case 2: return tiers ? batch_kernel<6, true, false> : batch_kernel<6, false, false>;
+    default: return tiers ? batch_kernel<0, true, false> : batch_kernel<0, false, false>;
+    }
 }
 
 const void *batch_kernel_variant(int variant, bool tiers, bool mips)

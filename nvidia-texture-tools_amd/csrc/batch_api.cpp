@@ -569,6 +569,7 @@ NTX_API ntx_status ntx_hip_batch_autotune(ntx_hip_batch *b, int reps, ntx_batch_
     // Coordinate descent: each field in turn over its candidates, others
     // fixed; the schedule first, the decomposition under it after.
     for (int field : { 6, 0, 1, 2, 3, 4, 5 }) {
+        if (field == 0 && best.schedule == 1) continue;  // one instance for every variant
         std::vector<int> cand;
         switch (field) {
         case 6: cand = { 0, 1 }; break;                             // schedule
