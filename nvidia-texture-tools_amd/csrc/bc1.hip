@@ -262,89 +262,159 @@ __device__ __forceinline__ void search_lane(const LaneImage &im, int blk, bool l
     }
 }
 
-// Lanes per block of each list, log2 in two bits per colour count.
-__device__ __forceinline__ int list_shift(uint64_t shifts, int k) { return int(shifts >> (2 * k)) & 3; }
+// Wavefronts of a search workgroup: with the term tables they fill a compute
+// unit's LDS (two wavefronts a SIMD, at their registers the most there are).
+constexpr int kSearchWaves = 8;
 
-// A way to cut the lists into wavefronts: the lanes per block that bring the
-// candidates a lane walks, C(n + 3, 3) of a list's blocks over its lanes, to
-// at most a limit (eight lanes at most), and what a wavefront of each list
-// then costs, in trips of a candidate (a block's set-up about 60).
-struct ListCut {
-    uint64_t shifts = 0;
-    int cost[17] = {};
+// A search's lists cut into wavefronts: of each list the first entries into
+// wavefronts of 64 >> s blocks, the others into finer ones.  The lists are
+// walked from count 16 down, first the coarse wavefronts, whole rounds of the
+// grid's, then the finer ones: one long wavefront too many would take as long
+// as a round, short ones fill in (blocks of 16 random texels, 65,536 and
+// 262,144 of them: 339 and 889 us with one cut for all, 266 and 716 so).
+//
+// Runs 0 to 14 are the coarse wavefronts of lists 16 to 2, 15 to 29 the finer
+// ones.
+constexpr int kRuns = 30;
+struct ListRuns {
+    int start[32];  // first wavefront
+    int first[32];  // first entry
+    int list[32];   // list | s << 8
+    int count[32];  // entries of the list
+    int total;      // wavefronts
+    float end[32];
 };
-constexpr ListCut cut_lists(int most)
+
+// How long a wavefront of list n at 1 << s lanes per block takes, in trips of
+// a candidate: both fits' and the set-up.
+constexpr int wave_trips(int n, int s)
 {
-    ListCut cut;
-    for (int n = 2; n <= 16; n++) {
-        int s = 0;
-        while (s < 3 && (n + 1) * (n + 2) * (n + 3) / 6 > most << s) s++;
-        cut.shifts |= uint64_t(s) << (2 * n);
-        cut.cost[n] = 60;
-        for (int b = 0; b <= n; b++) cut.cost[n] += ((b >> s) + 1) * (n - (b > 1 ? b : 1) + 1);
-    }
-    return cut;
+    int t = 120;
+    for (int b = 0; b <= n; b++) t += ((b >> s) + 1) * (n - (b > 1 ? b : 1) + 1 + (b > 0 ? 1 : 0));
+    return t;
+}
+struct TripTable {
+    uint16_t t[17][4] = {};
+};
+constexpr TripTable trip_table()
+{
+    TripTable r;
+    for (int n = 2; n <= 16; n++)
+        for (int s = 0; s < 4; s++) r.t[n][s] = uint16_t(wave_trips(n, s));
+    return r;
+}
+__device__ constexpr TripTable kTrips = trip_table();
+
+// The value of the lane N places before in the row of 16 (DPP row_shr), 0 in
+// the first N.
+template <int N, class V>
+__device__ __forceinline__ V row_before(V v)
+{
+    const int x = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x110 + N, 0xf, 0xf, false);
+    return __builtin_bit_cast(V, x);
+}
+__device__ __forceinline__ int row_before_sum(int v)  // of the lanes before
+{
+    const int own = v;
+    v += row_before<1>(v);
+    v += row_before<2>(v);
+    v += row_before<4>(v);
+    v += row_before<8>(v);
+    return v - own;
+}
+template <class V, class F>
+__device__ __forceinline__ V row_all(V v, F f)
+{
+    v = f(v, gror<8>(v));
+    v = f(v, gror<4>(v));
+    v = f(v, gror<2>(v));
+    return f(v, gror<1>(v));
 }
 
-// The cut of these lists for a grid of `slots` wavefronts, two a SIMD, that
-// should end first.  A wavefront alone on its SIMD takes 1.5 times as long a
-// trip as two side by side do between them, so the end is the longest
-// wavefront's or, where there is more to do, the sum's; and with more than a
-// few wavefronts in a second round not before about 900 trips (200 us), their
-// set-up coming after the first round's shortest.  Measured over noise and
-// rectangles at limits 130, 180, 250, 350, 500, 700 and none (us, the whole
-// call): 36,864 blocks 178, 132, 139, 166, 199, 257, 319; 43,264 blocks 202,
-// 203, 145, 168, 196; 65,536 blocks 217, 221, 151, 177, 198, 256, 341; 131,044
-// blocks 393, 391, 278, 294, 215, 270, 360; 262,144 blocks 760, 707, 529, 540,
-// 447, 459, 388.
-__device__ __forceinline__ uint64_t choose_cut(const int *__restrict__ counts, int cap, int slots)
+// The runs that should end first on a grid of `slots` wavefronts, two a SIMD,
+// the same in every workgroup; the whole workgroup of eight wavefronts calls
+// it, a row of 16 lanes a way to cut, a lane a list.  A way: the candidates
+// that a lane of a coarse wavefront walks at most, C(n + 3, 3) over its
+// block's lanes (eight at most), and the finer wavefronts' least lanes.
+//
+// A trip takes the same 0.24 us however many wavefronts a SIMD has, one or
+// two, and however many lanes a block: scheduling wavefronts of wave_trips so
+// comes within 8% of the measured times of five contents (noise with
+// rectangles, random texels, gradients, four colours a block, dark texels) at
+// 13 sizes and seven cuts each, and the estimate of the end below chooses as
+// that schedule would.  (A rule fitted to the first of these contents chose
+// cuts up to 1.2 times as long for the others.)
+__device__ __forceinline__ void choose_runs(ListRuns &runs, const int *__restrict__ counts, int cap, int slots)
 {
-    constexpr ListCut kCuts[] = { cut_lists(1 << 20), cut_lists(700), cut_lists(500), cut_lists(350),
-                                  cut_lists(250),     cut_lists(180), cut_lists(130) };
-    int c[17];
-#pragma unroll
-    for (int b = 2; b <= 16; b++) c[b] = min(counts[b], cap);
-    uint64_t pick = 0;
-    float least = FLT_MAX;
-#pragma unroll
-    for (int i = 0; i < 7; i++) {
-        int waves = 0, longest = 0;
-        float sum = 0.0f;
-#pragma unroll
-        for (int b = 2; b <= 16; b++) {
-            const int log2 = 6 - int(kCuts[i].shifts >> (2 * b) & 3);
-            const int wv = (c[b] + (1 << log2) - 1) >> log2;
-            waves += wv;
-            sum += float(wv) * float(kCuts[i].cost[b]);
-            if (wv > 0) longest = max(longest, kCuts[i].cost[b]);
-        }
-        const float end = fmaxf(fmaxf(1.5f * float(longest), sum / (0.5f * float(slots))),
-                                waves > slots + slots / 256 ? 900.0f : 0.0f);
-        if (end < least) {
-            least = end;
-            pick = kCuts[i].shifts;
-        }
+    static_assert(kSearchWaves == 8, "32 rows, a way each");
+    const int t = threadIdx.x, way = t >> 4, l = t & 15, n = 16 - l, m = way >> 2;
+    const int c = n >= 2 ? min(counts[n], cap) : 0;
+    const int most = m == 0 ? 1 << 20 : m == 1 ? 700 : m == 2 ? 500 : m == 3 ? 350 : m == 4 ? 250 : m == 5 ? 180 : 130;
+    const int each = (n + 1) * (n + 2) * (n + 3) / 6;
+    const int s = (each > most ? 1 : 0) + (each > 2 * most ? 1 : 0) + (each > 4 * most ? 1 : 0), f = max(s, way & 3);
+    const float trips = float(kTrips.t[n][s]), fine_trips = float(kTrips.t[n][f]);
+    const auto add = [](auto a, auto b) { return a + b; };
+    const auto greater = [](float a, float b) { return fmaxf(a, b); };
+
+    const int waves = (c + (64 >> s) - 1) >> (6 - s);
+    const int rounds = row_all(waves, add) / slots, coarse = rounds * slots;
+    const int before = min(row_before_sum(waves), coarse), k = min(waves, coarse - before);
+    const int done = min(k << (6 - s), c);
+    const int r = (c - done + (64 >> f) - 1) >> (6 - f);
+    const int rest = row_all(r, add);
+    const float sum = row_all(float(k) * trips, add), rest_sum = row_all(float(r) * fine_trips, add);
+    const float longest = row_all(k > 0 ? trips : 0.0f, greater), rest_longest = row_all(r > 0 ? fine_trips : 0.0f, greater);
+    // The first and the last wavefront of the last coarse round.
+    const float top = row_all(before <= coarse - slots && coarse - slots < before + k ? trips : 0.0f, greater);
+    const float last = row_all(k > 0 && before + k == coarse ? trips : 0.0f, greater);
+    const float per = 1.0f / float(slots), spread = fmaxf(top - last, 0.0f);
+    float end;
+    if (rounds == 0) {
+        end = rest <= slots ? fmaxf(rest_longest, rest_sum * per) : FLT_MAX;
+    } else if (rest == 0) {
+        end = fmaxf(longest, sum * per + (rounds > 1 ? 0.5f * spread : 0.0f));
+    } else {
+        // After coarse wavefronts that end together the finer ones take whole
+        // rounds; they fill in between those that end apart.
+        const float u = fminf(1.0f, spread / rest_longest);
+        const float whole = float((rest + slots - 1) / slots) * rest_longest;
+        end = fmaxf(longest, (sum + rest_sum) * per + (1.0f - u) * (whole - rest_sum * per) + u * 0.5f * rest_longest);
     }
-    return pick;
+    if (l == 0) runs.end[way] = way < 28 ? end : FLT_MAX;
+    __syncthreads();
+    const float own = runs.end[t & 31];
+    float least = own;
+#pragma unroll
+    for (int x = 1; x < 32; x <<= 1) least = fminf(least, __shfl_xor(least, x));
+    const int pick = __builtin_ctzll(__builtin_amdgcn_ballot_w64(own == least));
+    if (way == pick && l < 15) {
+        runs.start[l] = before;
+        runs.first[l] = 0;
+        runs.list[l] = n | s << 8;
+        runs.start[15 + l] = coarse + row_before_sum(r);
+        runs.first[15 + l] = done;
+        runs.list[15 + l] = n | f << 8;
+        runs.count[l] = runs.count[15 + l] = c;
+        if (l == 0) runs.total = coarse + rest;
+    }
+    __syncthreads();
 }
 
-// The wave-th wavefront of a search over lists cut into runs of 64 >> shift
-// entries: entries first .. of list k, the lists walked from count 16 down.
-// False past the last wavefront.
-__device__ __forceinline__ bool list_wave(const int *__restrict__ counts, int cap, uint64_t shifts, int wave, int &k,
-                                          int &first, int &cnt)
+// Wavefront `wave` of the runs: entries first .. of list k's cnt, 64 >> shift
+// of them.  False past the last wavefront.
+__device__ __forceinline__ bool list_wave(const ListRuns &runs, int wave, int lane, int &k, int &first, int &cnt, int &shift)
 {
-    int wv = wave;
-    k = 0;
-    for (int b = 16; b >= 2; b--) {
-        const int c = min(counts[b], cap), log2 = 6 - list_shift(shifts, b);
-        const int waves = (c + (1 << log2) - 1) >> log2;
-        if (k == 0) {
-            if (wv < waves) { k = b; first = wv << log2; cnt = c; }
-            else wv -= waves;
-        }
-    }
-    return k != 0;
+    if (wave >= __builtin_amdgcn_readfirstlane(runs.total)) return false;
+    // The last run that starts no later: those after it without wavefronts start later.
+    const int at = runs.start[lane & 31];
+    const int j = 63 - __builtin_clzll(__builtin_amdgcn_ballot_w64(lane < kRuns && at <= wave));
+    const int list = __builtin_amdgcn_readfirstlane(runs.list[j]);
+    k = list & 0xff;
+    shift = list >> 8;
+    cnt = __builtin_amdgcn_readfirstlane(runs.count[j]);
+    first = __builtin_amdgcn_readfirstlane(runs.first[j]) +
+            ((wave - __builtin_amdgcn_readfirstlane(runs.start[j])) << (6 - shift));
+    return true;
 }
 
 // Images of a search launch: `get` gives the image and block of a list
@@ -409,9 +479,6 @@ struct ImageSet {
     }
 };
 
-// Wavefronts of a search workgroup: with the term tables they fill a compute
-// unit's LDS (two wavefronts a SIMD, at their registers the most there are).
-constexpr int kSearchWaves = 8;
 
 // Level8 pass 2 (icbc.h:3292-3326 + :3543-3550).  The lists are cut into
 // wavefronts of consecutive entries, 1 to 8 lanes a block by list, and walked
@@ -433,16 +500,16 @@ __global__ __launch_bounds__(64 * kSearchWaves, 2) void bc1_search_kernel(Images
     __shared__ float4 s_rows[kSearchWaves][17][64];
     __shared__ SearchTables s_tables;
     __shared__ typename Images::Shared s_images;
+    __shared__ ListRuns s_runs;
     load_search_tables(s_tables, tab, threadIdx.x, 64 * kSearchWaves);
     images.load(s_images);
-    const uint64_t shifts = choose_cut(counts, cap, int(gridDim.x) * kSearchWaves);
-    __syncthreads();
+    choose_runs(s_runs, counts, cap, int(gridDim.x) * kSearchWaves);
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
     for (int wave = blockIdx.x + gridDim.x * wv;;) {
-        int k = 0, first = 0, cnt = 0;
-        if (!list_wave(counts, cap, shifts, wave, k, first, cnt)) break;
-        const int shift = list_shift(shifts, k), cols = 64 >> shift;
+        int k = 0, first = 0, cnt = 0, shift = 0;
+        if (!list_wave(s_runs, wave, lane, k, first, cnt, shift)) break;
+        const int cols = 64 >> shift;
         const int item = first + (lane & (cols - 1));
         bool live = item < cnt;
         // Every caller's lists hold blocks of its images; anything else is

@@ -219,6 +219,23 @@ def test_search_forms_match_one_pass(lanes, side, kind):
     assert _both_encoders(lanes, np.ascontiguousarray(img[:, :h]), w, h, **kw) == 0
 
 
+@pytest.mark.parametrize("kind", ["random", "dark", "few", "both"])
+@pytest.mark.parametrize("size", [(36, 28), (64, 64), (252, 260), (256, 256), (512, 132), (1024, 1024), (1448, 1452)])
+def test_search_cuts_by_content(lanes, kind, size):
+    """Lists that fill the grid's wavefronts exactly, by less, and by a block
+    more (one list of 16 colours, with a few shorter ones; four colours a
+    block; both): every block in exactly one wavefront, coarse or fine."""
+    w, h = size
+    rng = np.random.default_rng(w + h)
+    img = np.ones((4, h, w), np.float32)
+    img[:3] = rng.integers(0, 24 if kind == "dark" else 256, (3, h, w)) / np.float32(255)
+    if kind in ("few", "both"):
+        pal = (rng.integers(0, 256, (4, 3)) / 255).astype(np.float32)
+        few = pal[rng.integers(0, 4, (h, w))].transpose(2, 0, 1)
+        img[:3, :, w // 2 if kind == "both" else 0:] = few[:, :, w // 2 if kind == "both" else 0:]
+    assert _both_encoders(lanes, img, w, h) == 0
+
+
 @pytest.mark.parametrize("side", [60, 1024])
 @pytest.mark.parametrize("scale, alpha", [(s, 1.0) for s in (1e8, 3e9, 1e10, 1e14, 9e17)] +
                          [(1.0, a) for a in (1e-12, 1e-16, 1e-20, 1e-30)] + [(1e10, 1e-20)])
@@ -308,7 +325,7 @@ def test_optional_scratch_is_off_a_later_limit():
     """Calls that took the two-pass encoder's optional scratch leave a limit
     that is set afterwards to the calls that need theirs."""
     with N.Context(0) as ctx:
-        w, h = 1000, 917
+        w, h = 1280, 1232  # 98,560 blocks
         _, d = _input(ctx, w, h, 81)
         _, d2 = _input(ctx, 640, 480, 82)
         out = [ctx.alloc(N.compressed_size(N.FORMAT_BC1, a, b)) for a, b in ((w, h), (640, 480))]
@@ -333,9 +350,9 @@ def test_optional_scratch_and_recorded_graphs():
     with N.Context(0) as ctx:
         w, h = 128, 96
         _, d = _input(ctx, w, h, 91)
-        _, big = _input(ctx, 1000, 917, 92)
+        _, big = _input(ctx, 1280, 1232, 92)
         out = ctx.alloc(N.compressed_size(N.FORMAT_BC3, w, h))
-        out_big = ctx.alloc(N.compressed_size(N.FORMAT_BC1, 1000, 917))
+        out_big = ctx.alloc(N.compressed_size(N.FORMAT_BC1, 1280, 1232))
         ctx.compress_device(N.FORMAT_BC3, d, w, h, out)  # its scratch is there before the recording
         want = out.download(np.uint8)
         with _Capture(ctx, ctx.lib.ntx_hip_stream(ctx.handle), 2) as g:
@@ -347,9 +364,9 @@ def test_optional_scratch_and_recorded_graphs():
         for k in range(4):
             if k == 1:
                 with recording:
-                    ctx.compress_device(N.FORMAT_BC1, big, 1000, 917, out_big)
+                    ctx.compress_device(N.FORMAT_BC1, big, 1280, 1232, out_big)
             elif k > 1:
-                ctx.compress_device(N.FORMAT_BC1, big, 1000, 917, out_big)
+                ctx.compress_device(N.FORMAT_BC1, big, 1280, 1232, out_big)
             if k:
                 results.append(out_big.download(np.uint8))
             out.upload(np.zeros_like(want))
@@ -357,7 +374,7 @@ def test_optional_scratch_and_recorded_graphs():
             ctx.synchronize()
             assert np.array_equal(out.download(np.uint8), want), k
         ctx.set_bc1_lanes_min(1 << 30)
-        ctx.compress_device(N.FORMAT_BC1, big, 1000, 917, out_big)
+        ctx.compress_device(N.FORMAT_BC1, big, 1280, 1232, out_big)
         for r in results:
             assert np.array_equal(r, out_big.download(np.uint8))
         g.close()
