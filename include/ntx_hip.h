@@ -204,8 +204,9 @@ NTX_API ntx_status ntx_hip_set_scratch_limit(ntx_hip_context *ctx, size_t bytes)
  * least `min_blocks` 4x4 blocks, two passes with 1 to 8 lanes per block
  * (colour counts, then the cluster fit over blocks bucketed by count).  Sets
  * the context's threshold; 0 restores the default (2^17 blocks, and below
- * that from 53,248 blocks where its scratch is to be had: not under a scratch
- * limit or while the stream records a graph).  No counterpart in the
+ * that from 98,304 blocks, or 81,920 over a set of images, where its scratch
+ * is to be had: not under a scratch limit or while the stream records a
+ * graph).  No counterpart in the
  * reference. */
 NTX_API ntx_status ntx_hip_set_bc1_lanes_min(ntx_hip_context *ctx, int min_blocks);
 

@@ -165,13 +165,20 @@ struct ntx_hip_context {
     // Unless that threshold was set: an image of fewer blocks, but at least
     // this many, or a set of images of at least that many together, takes the
     // two-pass encoder too where its scratch is free to be had
-    // (optional_bc1_bucket), and the one-pass one otherwise.  One-pass and
-    // two-pass calls on noise and rectangles: 43,264 blocks 130 and 145 us,
-    // 50,176 blocks 146 and 146, 57,600 blocks 157 and 148, 65,536 blocks 201
-    // and 151, 131,044 blocks 322 and 213.  A 1000x750 chain (62,600 blocks,
-    // its levels in one launch either way) 187 and 195, a 1024^2 one (87,400)
-    // 288 and 240.
-    static constexpr int kBc1LanesOptional = 52 << 10, kBc1LanesOptionalSet = 72 << 10;
+    // (optional_bc1_bucket), and the one-pass one otherwise.  Which is faster
+    // lies with the content, which the host does not know: the lines are where
+    // no content measured takes more than 1.02 times what images of their own
+    // launches took before there was a choice.  One-pass and two-pass calls in
+    // us, noise with rectangles, random texels, gradients, four colours a
+    // block, dark texels: 65,536 blocks 198 and 148, 224 and 266, 202 and 225,
+    // 76 and 74, 184 and 193; 82,944 blocks 221 and 212, 282 and 326, 253 and
+    // 246, 97 and 80, 240 and 303; 102,400 blocks 259 and 199, 339 and 356, 304
+    // and 285, 115 and 85, 285 and 302; 131,044 blocks 291 and 212, 429 and 363,
+    // 386 and 322, 148 and 100, 363 and 374.  Chains of 74,261 blocks, one
+    // launch either way: 191 and 174, 257 and 299, 231 and 246, 105 and 85, 220
+    // and 283; of 87,383: 265 and 205, 302 and 331, 272 and 258, 122 and 84, 257
+    // and 311.
+    static constexpr int kBc1LanesOptional = 96 << 10, kBc1LanesOptionalSet = 80 << 10;
     // The BC3 tallies at the start of `bucket` are zero: set after a complete
     // front + search sequence (the search clears them), cleared before one.
     bool bc3_counts_zero = false;
