@@ -566,11 +566,17 @@ namespace ntx {
 
 // Groups per block of an image of `blocks` blocks: a block on one group
 // searches up to 61 runs of partitions one after another (about 37 us), which
-// an image that leaves SIMDs idle should not wait for: a 64^2 image (256
-// blocks) takes 37.4 us a call on one group a block, 14.4 us on sixteen.
+// an image that leaves SIMDs idle should not wait for.  Every group of a block
+// prepares it again, so the lines are where blocks of few colours, which have
+// next to nothing to search, lose no more than 2 us.  On 1, 4 and 16 groups,
+// noise with rectangles and blocks of four colours: 256 blocks 34.5, 18.1 and
+// 14.2 us, 13.8, 12.9 and 13.0; 400 blocks 35.6, 18.3 and 15.9, 14.1, 12.9 and
+// 14.8; 784 blocks 35.2, 18.3 and 21.0, 14.0, 13.1 and 21.0; 2,025 blocks 35.5,
+// 19.9 and 38.8, 13.5, 15.0 and 37.0; 4,096 blocks 35.4, 30.3 and 71.2, 13.6,
+// 21.7 and 68.1.
 static int bc1_parts(int blocks)
 {
-    return blocks <= 512 ? 16 : blocks <= 4096 ? 4 : 1;
+    return blocks <= 512 ? 16 : blocks <= 2048 ? 4 : 1;
 }
 
 // Up to kBc1MaxImages images in one launch, in the order given (the largest

@@ -220,11 +220,14 @@ def test_search_forms_match_one_pass(lanes, side, kind):
 
 
 @pytest.mark.parametrize("kind", ["random", "dark", "few", "both"])
-@pytest.mark.parametrize("size", [(36, 28), (64, 64), (252, 260), (256, 256), (512, 132), (1024, 1024), (1448, 1452)])
+@pytest.mark.parametrize("size", [(36, 28), (64, 64), (128, 64), (128, 68), (256, 128), (256, 132), (252, 260), (256, 256),
+                                  (512, 132), (1024, 1024), (1448, 1452)])
 def test_search_cuts_by_content(lanes, kind, size):
     """Lists that fill the grid's wavefronts exactly, by less, and by a block
     more (one list of 16 colours, with a few shorter ones; four colours a
-    block; both): every block in exactly one wavefront, coarse or fine."""
+    block; both): every block in exactly one wavefront, coarse or fine.  On
+    the other side sixteen, four (from 513 blocks) and one (from 2,049) groups
+    a block."""
     w, h = size
     rng = np.random.default_rng(w + h)
     img = np.ones((4, h, w), np.float32)
