@@ -151,25 +151,26 @@ __device__ __forceinline__ void fused_x_pass(const float *s_src, float *s_tmp, c
 #pragma unroll
             for (int j = 0; j < N; ++j) sum += kxr[j] * q[j];
         } else {
+            const float *row = s_src + r * kSrcW + xoff;
 #pragma unroll
             for (int j = 0; j < kMaxWin; ++j)
-                if (j < wx) sum += kxr[j] * (j & 1 ? odd_taps : even_taps)[r * kSrcW + j / 2];
+                if (j < wx) sum += kxr[j] * row[j];
         }
         s_tmp[r * kTX + xi] = sum;
     }
 }
 
 // A wavefront's output rows o0, o0 + 1 (those below ny): first rows f0, f1 of
-// s_tmp, weights k0, k1 (uniform).  Two rows of exactly N taps whose first
-// rows are two apart, as downsampling by about two has them, share their
-// reads: N + 2 instead of 2N.
+// s_tmp, weights k0, k1 (uniform).  Two rows whose first rows are two apart,
+// as downsampling by about two has them, share their reads: N + 2 instead of
+// 2N.
 template <int N>
 __device__ __forceinline__ void fused_y_pass(const float *s_tmp, const float *__restrict__ k0,
-                                             const float *__restrict__ k1, int f0, int f1, int wy, bool second, float &sum0, float &sum1)
+                                             const float *__restrict__ k1, int f0, int f1, bool second, float &sum0, float &sum1)
 {
     sum0 = sum1 = 0.0f;
     const float *c0 = s_tmp + f0 * kTX, *c1 = s_tmp + f1 * kTX;
-    if (N > 0 && second && f1 == f0 + 2) {
+    if (second && f1 == f0 + 2) {
         float q[N + 2];
 #pragma unroll
         for (int j = 0; j < N + 2; ++j) q[j] = c0[j * kTX];
@@ -180,14 +181,11 @@ __device__ __forceinline__ void fused_y_pass(const float *s_tmp, const float *__
         }
         return;
     }
-    constexpr int kTaps = N > 0 ? N : kMaxWin;
 #pragma unroll
-    for (int j = 0; j < kTaps; ++j)
-        if (N > 0 || j < wy) sum0 += k0[j] * c0[j * kTX];
+    for (int j = 0; j < N; ++j) sum0 += k0[j] * c0[j * kTX];
     if (!second) return;
 #pragma unroll
-    for (int j = 0; j < kTaps; ++j)
-        if (N > 0 || j < wy) sum1 += k1[j] * c1[j * kTX];
+    for (int j = 0; j < N; ++j) sum1 += k1[j] * c1[j * kTX];
 }
 
 // kPair: every output's first tap is two source columns after its left
@@ -196,11 +194,12 @@ __device__ __forceinline__ void fused_y_pass(const float *s_tmp, const float *__
 // (consecutive lanes on consecutive 8-byte words: no bank conflicts).
 // kWinX, kWinY > 0: the passes have exactly that many taps, known when
 // compiling, so the tap loops unroll without a test per tap and a window's
-// reads travel together; 0: wx and wy taps as passed.
+// reads travel together; 0, both: wx and wy taps as passed, a test for each
+// (its loads, weights too, then come one after another: what the window does
+// not need is not loaded, and the Y weights are staged).
 // kUni: exact halving with the same taps for every output (kPair, windows > 0):
 // the weights come from `taps` and output i's first tap is l0 + 2 i, so no
 // table is read before the staging loads (small levels are latency-bound).
-// Six waves per SIMD are what the LDS of its workgroups admits.
 // Six waves per SIMD are what the LDS of its workgroups admits; with 14 taps in
 // registers five are as fast (48 against 50 us, the sixth's registers spill).
 template <bool kPair, int kWinX, int kWinY, bool kUni = false>
@@ -213,12 +212,16 @@ void poly_fused_kernel(const float *__restrict__ src, int W, int H,
 {
     static_assert(2 * (kTX - 1) + kMaxWin <= kSrcW, "paired X reads stay inside a staged row");
     static_assert(kWinX >= 0 && kWinX <= kMaxWin && kWinY >= 0 && kWinY <= kMaxWin, "window held in registers");
+    static_assert((kWinX > 0) == (kWinY > 0), "both windows are known, or neither");
     static_assert(!kUni || (kPair && kWinX > 0 && kWinY > 0), "uniform taps: exact halving of a fixed window");
     static_assert(kTY == 2 * kWaves, "two output rows a wavefront");
     if (kWinX > 0) wx = kWinX;
     if (kWinY > 0) wy = kWinY;
     __shared__ __align__(16) float s_src[kSrcH * kSrcW];
     __shared__ float s_tmp[kSrcH * kTX];
+    static_assert(kTY * kMaxWin <= 64 * kWaves, "one thread per staged Y weight");
+    __shared__ float s_ky[kWinY == 0 ? kTY * kMaxWin : 1];
+    __shared__ int s_ly[kWinY == 0 ? kTY : 1];
     const int t = threadIdx.x;
     int tX, tY;
     tile_coords(blockIdx.x, tx, tX, tY);
@@ -237,7 +240,7 @@ void poly_fused_kernel(const float *__restrict__ src, int W, int H,
         xoff = kPair ? 2 * xi : lx[ox0 + xi] - cx0;
         const float *k = kUni ? taps.kx : kx + size_t(ox0 + xi) * wx;
 #pragma unroll
-        for (int j = 0; j < kMaxWin; j++) kxr[j] = kUni ? taps.kx[j] : k[min(j, wx - 1)];
+        for (int j = 0; j < kMaxWin; j++) kxr[j] = kUni ? taps.kx[j] : j < wx ? k[j] : 0.0f;
     }
 
     // The wavefront's two output rows: weights and first rows of s_tmp, the
@@ -255,6 +258,14 @@ void poly_fused_kernel(const float *__restrict__ src, int W, int H,
         ky1 = ky + size_t(y1) * wy;
     }
 
+    if (kWinY == 0) {
+        if (t < ny * kMaxWin) {
+            const int o = t / kMaxWin, j = t % kMaxWin;
+            s_ky[t] = j < wy ? ky[size_t(oy0 + o) * wy + j] : 0.0f;
+        }
+        if (t < ny) s_ly[t] = ly[oy0 + t] - ry0;
+    }
+
     // Staging: lane (t & 63) owns source columns (t & 63) + 64k of the tile,
     // whose wrapped image columns are fixed; wave (t >> 6) owns rows
     // (t >> 6) + kWaves i.  A plane's loads are all issued before its LDS stores
@@ -269,7 +280,7 @@ void poly_fused_kernel(const float *__restrict__ src, int W, int H,
     for (int k = 0; k < kColSlots; k++) {
         const int col = xi + kTX * k;
         cvalid[k] = col < sw;
-        at[k] = kPair ? col : split_column(col);
+        at[k] = kPair || kWinX == 0 ? col : split_column(col);
         gx[k] = wrap_index(cx0 + (cvalid[k] ? col : 0), W, wrap);
     }
     size_t rowoff[kRowSlots];
@@ -310,10 +321,20 @@ void poly_fused_kernel(const float *__restrict__ src, int W, int H,
         }
         if (xlive) fused_x_pass<kPair, kWinX>(s_src, s_tmp, kxr, xi, xoff, wx, wave, sh);
         __syncthreads();
-        if (xlive && o0 < ny) {
+        if constexpr (kWinY == 0) {
+            float *out = dst + size_t(c) * size_t(w) * size_t(h);
+            for (int o = wave; xlive && o < ny; o += kWaves) {
+                const float *k = s_ky + o * kMaxWin;
+                const float *col = s_tmp + s_ly[o] * kTX + xi;
+                float sum = 0.0f;
+#pragma unroll
+                for (int j = 0; j < kMaxWin; ++j)
+                    if (j < wy) sum += k[j] * col[j * kTX];
+                out[size_t(oy0 + o) * size_t(w) + ox0 + xi] = sum;
+            }
+        } else if (xlive && o0 < ny) {
             float sum0, sum1;
-            const float *col = s_tmp + xi;
-            fused_y_pass<kWinY>(col, ky0, ky1, f0, f1, wy, second, sum0, sum1);
+            fused_y_pass<kWinY>(s_tmp + xi, ky0, ky1, f0, f1, second, sum0, sum1);
             float *out = dst + size_t(c) * size_t(w) * size_t(h) + size_t(oy0 + o0) * size_t(w) + ox0 + xi;
             out[0] = sum0;
             if (second) out[w] = sum1;

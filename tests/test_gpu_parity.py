@@ -198,6 +198,19 @@ def test_mip_windows_of_odd_sides(gpu, oracle, filt, wrap, size):
         assert np.array_equal(_bits(a), _bits(b)), width
 
 
+@pytest.mark.parametrize("width", [0.7, 1.5, 2.0, 2.5, 3.4])
+@pytest.mark.parametrize("size", [(128, 96), (301, 199), (129, 130), (2 * 65, 2 * 17 + 1), (259, 35)])
+def test_mip_windows_not_compiled_in(gpu, oracle, width, size):
+    """Windows of other widths than the filters' own: even and odd sides,
+    whole tiles of 64 x 16 outputs and one output more."""
+    W, H = size
+    planar = np.random.default_rng(W * 131 + H).standard_normal(4 * W * H).astype(np.float32)
+    for filt in (N.FILTER_BOX, N.FILTER_TRIANGLE):
+        a = gpu.downsample(filt, planar, W, H, width=width)
+        b = oracle.build_next_mipmap(filt, width, None, N.WRAP_MIRROR, planar, W, H)
+        assert np.array_equal(_bits(a), _bits(b)), filt
+
+
 @pytest.mark.parametrize("filt", [N.FILTER_BOX, N.FILTER_TRIANGLE, N.FILTER_KAISER])
 @pytest.mark.parametrize("wrap", [N.WRAP_CLAMP, N.WRAP_REPEAT, N.WRAP_MIRROR])
 @pytest.mark.parametrize("size", [(64, 64), (37, 23), (1, 7), (6, 1), (2, 2), (5, 4), (130, 66), (3, 3)])
