@@ -194,8 +194,8 @@ __device__ __forceinline__ float eval_from_sum(float axr, float axg, float axb, 
 
 // Half of eval_from_sum's error under the metric (1, 1, 1), from the terms
 // h = (alpha2 / 2, beta2 / 2, alphabeta / 2, 2 * factor): scaling by powers
-// of two commutes with every rounding on the way (bc1_tame keeps subnormal
-// values out), so 2 * the result is the same float, and the three doublings
+// of two commutes with every rounding on the way (tame_component and
+// Reduced::tame keep subnormal values out), so 2 * the result is the same float, and the three doublings
 // of the cross terms go.
 __device__ __forceinline__ float half_error_from_sum(float axr, float axg, float axb, float4 sum, float4 h,
                                                      Cand *out = nullptr)

@@ -133,7 +133,7 @@ def test_colour_counts_match_oracle(lanes, oracle):
 
 def test_two_encoders_agree_on_large_images(lanes, gpu):
     """1024^2 (65,536 blocks) and 2048x512, default context (one-pass below
-    2^17 blocks) against the two-pass context."""
+    98,304 blocks) against the two-pass context."""
     for (w, h, seed) in ((1024, 1024, 3), (2048, 512, 4)):
         planar = synth.to_planar(synth.noise_rect_rgba(w, h, seed=seed, transparent=seed == 4)).reshape(-1)
         for mode in (N.ALPHA_NONE, N.ALPHA_TRANSPARENCY):
@@ -263,9 +263,10 @@ def test_search_where_the_axis_overflows(lanes, oracle, side, scale, alpha):
 
 
 def test_default_route_by_size_and_scratch():
-    """A context as it is made: images and sets above the sizes where the
-    two-pass encoder is optional, with and without a scratch limit (which
-    keeps it off), give the one-pass encoder's bytes."""
+    """A context as it is made: a set of 87,710 blocks, where the two-pass
+    encoder is optional, with and without a scratch limit (which keeps it
+    off), and an image of 57,500, below the line for one, give the one-pass
+    encoder's bytes."""
     free, capped, one = N.Context(0), N.Context(0), N.Context(0)
     try:
         capped.lib.ntx_hip_set_scratch_limit(capped.handle, 1)
