@@ -152,8 +152,9 @@ __device__ __forceinline__ void classify_chunk(const float *__restrict__ src, in
 // block of one colour compress_dxt1_single_color_optimal (icbc.h:3515-3525),
 // every other block goes to list n.  The clusters live in LDS only while
 // they are counted.  (Clusters as three columns without weights, 48 KB a
-// workgroup and three wavefronts a SIMD, took 510 us at 8192^2 where this
-// takes 460: the LDS reads, one of 16 bytes here, are what it waits for.)
+// workgroup and three wavefronts a SIMD, took 510 us at 8192^2 where this took
+// 460, and takes 482: the LDS reads, one of 16 bytes here, are what it waits
+// for.)
 __global__ __launch_bounds__(256) void bc1_classify_kernel(const float *__restrict__ src, int w, int h, int bw, int nblocks,
                                                            int alpha_mode, const ntx::Tables *__restrict__ tab,
                                                            uint2 *__restrict__ out, short2 *__restrict__ nm,

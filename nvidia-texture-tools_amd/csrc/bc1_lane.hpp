@@ -58,22 +58,42 @@ struct BlockTexels {
     // weight = saturate(alpha) for Transparency, else 1.
     __device__ __forceinline__ void row(int r, float4 (&t)[4]) const
     {
+        if (whole) whole_row(r, t);
+        else edge_row(r, t);
+    }
+    // All rows, 4 r + i: one branch, so that every row's loads are in flight
+    // together (a branch a row, with a wait at its end: 8192^2 classified in
+    // 516 us, 482 so).
+    __device__ __forceinline__ void all(float4 (&t)[16]) const
+    {
         if (whole) {
-            const float *p = src + size_t(y + r) * size_t(w) + size_t(x);
-            const float4 vr = *reinterpret_cast<const float4 *>(p);
-            const float4 vg = *reinterpret_cast<const float4 *>(p + plane);
-            const float4 vb = *reinterpret_cast<const float4 *>(p + 2 * plane);
-            float4 wt = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-            if (transparency) {
-                const float4 va = *reinterpret_cast<const float4 *>(p + 3 * plane);
-                wt = make_float4(icbc_saturate(va.x), icbc_saturate(va.y), icbc_saturate(va.z), icbc_saturate(va.w));
-            }
-            t[0] = make_float4(vr.x, vg.x, vb.x, wt.x);
-            t[1] = make_float4(vr.y, vg.y, vb.y, wt.y);
-            t[2] = make_float4(vr.z, vg.z, vb.z, wt.z);
-            t[3] = make_float4(vr.w, vg.w, vb.w, wt.w);
+#pragma unroll
+            for (int r = 0; r < 4; r++) whole_row(r, t + 4 * r);
             return;
         }
+#pragma unroll
+        for (int r = 0; r < 4; r++) edge_row(r, t + 4 * r);
+    }
+
+private:
+    __device__ __forceinline__ void whole_row(int r, float4 *t) const
+    {
+        const float *p = src + (size_t(y) * size_t(w) + size_t(x)) + size_t(r) * size_t(w);  // r w: scalar
+        const float4 vr = *reinterpret_cast<const float4 *>(p);
+        const float4 vg = *reinterpret_cast<const float4 *>(p + plane);
+        const float4 vb = *reinterpret_cast<const float4 *>(p + 2 * plane);
+        float4 wt = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        if (transparency) {
+            const float4 va = *reinterpret_cast<const float4 *>(p + 3 * plane);
+            wt = make_float4(icbc_saturate(va.x), icbc_saturate(va.y), icbc_saturate(va.z), icbc_saturate(va.w));
+        }
+        t[0] = make_float4(vr.x, vg.x, vb.x, wt.x);
+        t[1] = make_float4(vr.y, vg.y, vb.y, wt.y);
+        t[2] = make_float4(vr.z, vg.z, vb.z, wt.z);
+        t[3] = make_float4(vr.w, vg.w, vb.w, wt.w);
+    }
+    __device__ __forceinline__ void edge_row(int r, float4 *t) const
+    {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -166,13 +186,7 @@ __device__ __forceinline__ int classify_reduce(LaneRows rows, int lane, const Bl
 {
     const float thr = 1.0f / 256;
     float4 t[16];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        float4 row[4];
-        texels.row(r, row);
-#pragma unroll
-        for (int i = 0; i < 4; i++) t[4 * r + i] = row[i];
-    }
+    texels.all(t);
     int n = 0;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
