@@ -194,9 +194,9 @@ NTX_API ntx_status ntx_hip_compress_device_noalloc(ntx_hip_context *ctx, int for
  * NTX_ERR_OUT_OF_MEMORY (Error_CudaError in the nvtt front end, which then
  * goes on with the next image, as CudaCompressorDXT.cpp:183-189 does).
  * Scratch that a call can do without (see ntx_hip_set_bc1_lanes_min) is given
- * back when a cap is set, after the work on the context's stream, and not
- * taken under one.  0 = no cap (the default).  No counterpart in the
- * reference. */
+ * back when a cap is set, after the work on the context's stream (not while
+ * that records a graph), and not taken under one.  0 = no cap (the default).
+ * No counterpart in the reference. */
 NTX_API ntx_status ntx_hip_set_scratch_limit(ntx_hip_context *ctx, size_t bytes);
 
 /* BC1 at icbc Level8 (Normal / Highest) has two encoders with identical
@@ -206,8 +206,7 @@ NTX_API ntx_status ntx_hip_set_scratch_limit(ntx_hip_context *ctx, size_t bytes)
  * the context's threshold; 0 restores the default (2^17 blocks, and below
  * that from 98,304 blocks, or 81,920 over a set of images, where its scratch
  * is to be had: not under a scratch limit or while the stream records a
- * graph).  No counterpart in the
- * reference. */
+ * graph).  No counterpart in the reference. */
 NTX_API ntx_status ntx_hip_set_bc1_lanes_min(ntx_hip_context *ctx, int min_blocks);
 
 /* BC1 only: also writes, per block, the colour count after reduce_colors (n)

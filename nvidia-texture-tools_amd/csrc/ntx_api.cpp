@@ -777,11 +777,20 @@ static ntx_status single_bucket(ntx_hip_context *ctx, int format, int quality, i
     return NTX_OK;
 }
 
+// Whether the context's stream records a graph (or cannot tell).
+static bool recording(ntx_hip_context *ctx)
+{
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+}
+
 // Gives the optional encoder's scratch back.  The searches that use it are on
-// the context's stream, and no graph holds it (optional_bc1_bucket).
+// the context's stream, and no graph holds it (optional_bc1_bucket).  While
+// the stream records it can neither be waited for nor the memory be used: it
+// stays.
 static hipError_t release_optional(ntx_hip_context *ctx)
 {
-    if (!ctx->optional.ptr) return hipSuccess;
+    if (!ctx->optional.ptr || recording(ctx)) return hipSuccess;
     const AnyCapture allow;
     hipError_t e = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) e = hipFree(ctx->optional.ptr);
@@ -796,10 +805,8 @@ static hipError_t release_optional(ntx_hip_context *ctx)
 static int *optional_bc1_bucket(ntx_hip_context *ctx, int quality, size_t blocks)
 {
     if (ctx->bc1_lanes_min != ntx_hip_context::kBc1LanesMinDefault || ctx->scratch_limit || bc1_level(quality) != 8 ||
-        blocks >= size_t(1) << 26)
+        blocks >= size_t(1) << 26 || recording(ctx))
         return nullptr;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
     const size_t bytes = sizeof(int) * size_t(bc1_scratch_ints(int(blocks)));
     if (ctx->optional.cap < bytes) {
         const AnyCapture allow;

@@ -348,9 +348,9 @@ def test_optional_scratch_is_off_a_later_limit():
 
 def test_optional_scratch_and_recorded_graphs():
     """A graph recorded over a call that needs the context's scratch, replayed
-    after calls that took the optional one and between others; and a call with
-    the optional scratch while another stream records, which the recording
-    survives."""
+    after calls that took the optional one and between others; a scratch limit
+    set while the context's stream records, and a call with the optional
+    scratch while another stream does, which the recordings survive."""
     with N.Context(0) as ctx:
         w, h = 128, 96
         _, d = _input(ctx, w, h, 91)
@@ -359,8 +359,13 @@ def test_optional_scratch_and_recorded_graphs():
         out_big = ctx.alloc(N.compressed_size(N.FORMAT_BC1, 1280, 1232))
         ctx.compress_device(N.FORMAT_BC3, d, w, h, out)  # its scratch is there before the recording
         want = out.download(np.uint8)
+        ctx.compress_device(N.FORMAT_BC1, big, 1280, 1232, out_big)
         with _Capture(ctx, ctx.lib.ntx_hip_stream(ctx.handle), 2) as g:
             ctx.compress_device(N.FORMAT_BC3, d, w, h, out)
+            for limit in (1 << 30, 0):
+                ctx.lib.ntx_hip_set_scratch_limit(ctx.handle, limit)
+        ctx.lib.ntx_hip_set_scratch_limit(ctx.handle, 1 << 30)
+        ctx.lib.ntx_hip_set_scratch_limit(ctx.handle, 0)
         other = ctypes.c_void_p()
         assert ctx.lib.hipStreamCreateWithFlags(ctypes.byref(other), 1) == 0
         recording = _Capture(ctx, other.value, 0)
