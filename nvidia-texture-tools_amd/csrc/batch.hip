@@ -327,8 +327,9 @@ void batch_kernel(BatchArgs a)
     }
 }
 
-// Clears the ready counters, the queue position and the status word (a
-// kernel rather than a memset node, so the run can be captured in a graph).
+// Clears ready counters, queue positions, tallies (a kernel rather than a
+// memset, which a captured graph would hold as a node of its own kind and the
+// null stream would run beside the context's).
 __global__ __launch_bounds__(256) void batch_reset_kernel(int *p, int n)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;

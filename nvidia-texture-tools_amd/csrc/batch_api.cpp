@@ -15,7 +15,6 @@
 
 namespace ntx {
 hipError_t launch_batch(const BatchArgs &args, int variant, bool tiers, bool mips, int workgroups, hipStream_t stream);
-hipError_t launch_batch_reset(int *p, int n, hipStream_t stream);
 hipError_t launch_batch_mips(const BatchArgs &args, hipStream_t stream);
 hipError_t batch_resident_workgroups(int device, int variant, bool tiers, bool mips, int *count);
 int batch_kernel_variants();
@@ -465,7 +464,7 @@ NTX_API ntx_status ntx_hip_batch_create(ntx_hip_context *ctx, const ntx_texture_
                 e = hipMemcpy(b->d_bc1_imgs, imgs.data(), sizeof(ntx::Bc1Image) * imgs.size(), hipMemcpyHostToDevice);
             if (e == hipSuccess) e = hipMemcpy(b->d_bc1_map, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice);
             // Tallies and tickets zero before the first run (the lists need no clearing).
-            if (e == hipSuccess) e = hipMemset(b->d_bc1_bucket, 0, sizeof(int) * size_t(ntx::bc3_lists_offset()));
+            if (e == hipSuccess) e = ntx::launch_batch_reset(b->d_bc1_bucket, ntx::bc3_lists_offset(), ctx->stream);
             if (e != hipSuccess) return cleanup(ntx::fail(ctx, e, "batch BC1 tables"));
         }
     }

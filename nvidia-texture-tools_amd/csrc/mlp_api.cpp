@@ -71,8 +71,8 @@ ntx_status upload_params(ntx_hip_mlp *m, const float *params)
     ntx_hip_context *ctx = m->ctx;
     const size_t bytes = sizeof(float) * ntx_mlp::kParams;
     NTX_HIP(ctx, hipMemcpy(m->d_params, params, bytes, hipMemcpyHostToDevice));
-    NTX_HIP(ctx, hipMemset(m->d_m1, 0, bytes));
-    NTX_HIP(ctx, hipMemset(m->d_m2, 0, bytes));
+    for (float *p : { m->d_m1, m->d_m2 })
+        NTX_HIP(ctx, ntx::launch_batch_reset(reinterpret_cast<int *>(p), ntx_mlp::kParams, ctx->stream));
     m->step = 0;
     return NTX_OK;
 }

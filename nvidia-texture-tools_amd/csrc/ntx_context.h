@@ -36,6 +36,8 @@ hipError_t launch_bc1_search_multi(const Bc1Image *d_imgs, int nimgs, const Tabl
 // searches: a grid-stride loop over the blocks.
 constexpr int kOptimalGroupsPerCU = 8;
 int bc1_scratch_ints(int nblocks);
+// Zeros n ints at p.
+hipError_t launch_batch_reset(int *p, int n, hipStream_t stream);
 hipError_t launch_bc1_classify_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, const Tables *d_tab,
                                    int *d_counts, int cap, hipStream_t stream);
 hipError_t launch_bc1_search_set(const Bc1Target *images, int n, int alpha_mode, const float *cw, const Tables *d_tab,
