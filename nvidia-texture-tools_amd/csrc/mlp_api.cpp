@@ -229,7 +229,7 @@ ntx_status mlp_compress_on(ntx_hip_mlp *m, hipStream_t stream, int *d_count, int
 {
     ntx_hip_context *ctx = m->ctx;
     const int n = ((w + 3) / 4) * ((h + 3) / 4);
-    NTX_HIP(ctx, hipMemsetAsync(d_count, 0, sizeof(int), stream));
+    NTX_HIP(ctx, ntx::launch_batch_reset(d_count, 1, stream));  // no memset: the caller may record a graph
     const int cus = resident_cus(ctx);
     hipError_t e = ntx::timed_on(ctx, stream, NTX_KERNEL_BC1_MLP, [&] {
         return ntx::launch_bc1_mlp(m->d_params, d_rgba, w, h, ctx->d_tab, tau_pred, tau_gap, refine_iters, greedy_rounds,

@@ -15,6 +15,7 @@ import pytest
 
 import blocks
 import ntx_amd as N
+from capture import Capture
 from ntx_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -295,31 +296,6 @@ def test_default_route_by_size_and_scratch():
             ctx.close()
 
 
-class _Capture:
-    """HIP stream capture through the library's own runtime: mode 0 global, 2 relaxed."""
-
-    def __init__(self, ctx, stream, mode):
-        self.lib, self.stream, self.graph, self.exec = ctx.lib, ctypes.c_void_p(stream), ctypes.c_void_p(), ctypes.c_void_p()
-        self.mode = mode
-
-    def __enter__(self):
-        assert self.lib.hipStreamBeginCapture(self.stream, self.mode) == 0
-        return self
-
-    def __exit__(self, *exc):
-        assert self.lib.hipStreamEndCapture(self.stream, ctypes.byref(self.graph)) == 0
-        if exc[0] is None and self.graph:
-            assert self.lib.hipGraphInstantiate(ctypes.byref(self.exec), self.graph, None, None, ctypes.c_size_t(0)) == 0
-
-    def launch(self):
-        assert self.lib.hipGraphLaunch(self.exec, self.stream) == 0
-
-    def close(self):
-        for f, h in ((self.lib.hipGraphExecDestroy, self.exec), (self.lib.hipGraphDestroy, self.graph)):
-            if h:
-                assert f(h) == 0
-
-
 def _input(ctx, w, h, seed):
     p = synth.to_planar(synth.noise_rect_rgba(w, h, seed=seed)).reshape(-1)
     return p, ctx.alloc(p.nbytes).upload(p)
@@ -360,7 +336,7 @@ def test_optional_scratch_and_recorded_graphs():
         ctx.compress_device(N.FORMAT_BC3, d, w, h, out)  # its scratch is there before the recording
         want = out.download(np.uint8)
         ctx.compress_device(N.FORMAT_BC1, big, 1280, 1232, out_big)
-        with _Capture(ctx, ctx.lib.ntx_hip_stream(ctx.handle), 2) as g:
+        with Capture(ctx, ctx.lib.ntx_hip_stream(ctx.handle), 2) as g:
             ctx.compress_device(N.FORMAT_BC3, d, w, h, out)
             for limit in (1 << 30, 0):
                 ctx.lib.ntx_hip_set_scratch_limit(ctx.handle, limit)
@@ -368,7 +344,7 @@ def test_optional_scratch_and_recorded_graphs():
         ctx.lib.ntx_hip_set_scratch_limit(ctx.handle, 0)
         other = ctypes.c_void_p()
         assert ctx.lib.hipStreamCreateWithFlags(ctypes.byref(other), 1) == 0
-        recording = _Capture(ctx, other.value, 0)
+        recording = Capture(ctx, other.value, 0)
         results = []
         for k in range(4):
             if k == 1:

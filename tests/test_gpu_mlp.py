@@ -13,6 +13,7 @@ from ntx_amd import learned, synth
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
 import mlp_ref as R  # noqa: E402
+from capture import Capture  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -311,3 +312,27 @@ def test_images_entry_matches_per_image_calls(gpu):
                 d.free()
     for d in d_lv:
         d.free()
+
+
+def test_recorded_call_replays():
+    """The proposals and their fallback recorded as a graph (the fallback's
+    count cleared inside it): every replay, with other eager calls of the
+    network between, gives the eager call's blocks."""
+    w, h = 256, 192
+    with N.Context(0) as ctx:
+        d, other = (ctx.alloc(16 * w * h).upload(_texture(w, h, s)) for s in (21, 22))
+        size = N.compressed_size(N.FORMAT_BC1, w, h)
+        out, scratch = ctx.alloc(size), ctx.alloc(size)
+        with N.Mlp(ctx, _random_params(4)) as net:
+            fb = net.compress_bc1_device(d, w, h, out, tau_pred=0.6)
+            assert 0 < fb < size // 8
+            want = out.download(np.uint8)
+            with Capture(ctx, ctx.lib.ntx_hip_stream(ctx.handle), 2) as g:
+                net.compress_bc1_device(d, w, h, out, tau_pred=0.6, count_fallback=False)
+            for k in range(4):
+                out.upload(np.zeros_like(want))
+                g.launch()
+                ctx.synchronize()
+                assert np.array_equal(out.download(np.uint8), want), k
+                net.compress_bc1_device(other, w, h, scratch, tau_pred=0.6)
+            g.close()
